@@ -421,3 +421,41 @@ def test_padding_rows_never_read_past_the_chunk(dev, oracle, half, last):
         cc, cs = oracle.chunk_rule_varlen(**inp, cu=cu)
         assert max_rel(gc, cc) <= TOL
         assert max_rel(gs, cs) <= TOL
+
+
+@pytest.mark.parametrize("seqs", [1, 5])  # 16- and 32-column workgroups of the fp16 scan (16 heads)
+def test_fp16_scan_scales_are_per_column(dev, oracle, seqs):
+    """The fp16 scan holds fp32 operands as scaled halves, one power of two per
+    value column: columns of an initial state that differ by 2^80 each keep
+    fp32-level accuracy, and an infinity in V changes nothing in the other
+    columns, in the same column's earlier 16-token blocks, or in other heads."""
+    from spock_amd import synth
+    H, T, D = 16, 150, 128
+    cu = synth.cu_seqlens_from([T] * seqs)
+    inp = synth.chunk_inputs(H, T * seqs, seed=31)
+    for n in ("q", "k", "v"):
+        inp[n] = inp[n].astype(np.float16).astype(np.float32)
+    rng = np.random.default_rng(3)
+    init = (rng.normal(0, 1, (seqs, H, D, D)) * 2.0 ** rng.integers(-40, 41, D)).astype(np.float32)
+    gc, gs = _run(dev, inp, init=init, cu=cu, half=True)
+    sub = {n: np.ascontiguousarray(a[:2, :T]) for n, a in inp.items()}
+    c64, s64 = oracle.delta_recurrence_f64(**sub, init=init[0, :2])
+    # the file's 1e-5 against each column's largest value.  Either form's error
+    # here is the decays': a running sum of 64 log-decays below 128 in size
+    # rounds by up to 2^-18 at each step, 8 x 2^-18 x 0.58 = 1.8e-5 (one
+    # standard deviation of the sum) at its end in the exponent, where the
+    # decayed term itself no longer counts
+    for g, e in ((gc[:2, :T], c64), (gs[0, :2], s64)):
+        top = np.abs(e).max(axis=1, keepdims=True)
+        assert np.max(np.abs(g - e) / top) <= TOL
+    # an infinity at token 100 (chunk 1, block 2) of head 1, column 37
+    bad = {n: a.copy() for n, a in inp.items()}
+    bad["v"][1, 100, 37] = np.inf
+    bc, bs = _run(dev, bad, init=init, cu=cu, half=True)
+    assert not np.isfinite(bc[1, 100, 37]) and not np.isfinite(bs[0, 1, :, 37]).any()
+    same = np.ones_like(gc, dtype=bool)
+    same[1, 96:T, 37] = False
+    assert np.array_equal(bc[same], gc[same])
+    same = np.ones_like(gs, dtype=bool)
+    same[0, 1, :, 37] = False
+    assert np.array_equal(bs[same], gs[same])
