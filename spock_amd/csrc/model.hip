@@ -774,6 +774,364 @@ __global__ __launch_bounds__(256) void attn_prefill_blocks_kernel(AttnArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Long prompts: the same sums on the fp32 matrix cores.
+//
+// v_mfma_f32_16x16x4_f32 adds its four products to C one after the other, k = 0
+// to 3, each with one rounding (checked against chains of fmaf on random
+// operands, subnormal results included: no difference), so a chain of them is
+// the sequential fma chain of the per-token kernels, bit for bit, at twice the
+// vector ALU's rate.  Three launches:
+//   attn_qkv_prep_kernel   q normed and roped once per token (the block kernel
+//                          above repeats it for every block), K/V rows stored
+//   attn_scores_kernel     q.k / 16 of 16 tokens x 64 positions per wavefront
+//                          (256 MFMA in four chains); the block's maximum and
+//                          weights of each row and their sum
+//   attn_pv_kernel         16 tokens of one head per workgroup: blocks in
+//                          order, the weighted V sum (64 MFMA per block and 64
+//                          dims), the running combine -- the
+//                          maximum over all blocks is known beforehand, so the
+//                          blocks' partial outputs stay in registers instead of
+//                          going through memory (1 KB per token, head and
+//                          block; the weights are 256 B)
+// Bound by the matrix issue of 32 cycles per instruction (2,000 tokens: 56 us of
+// it in each of the last two launches, which take 106 and 127 us), by the
+// score launches' prologues and by the longest tile's chain of blocks.
+// Attention layer prefill, projections included: 512 tokens 122 -> 89 us, 1,000
+// 318 -> 136, 2,000 1,108 -> 318, 500 at position 1,000 251 -> 141.
+// ---------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kAttnRows = 16;  // tokens per tile
+// The tiles serve prompts of at least kAttnTileTokens tokens (below, few tiles
+// wait for a long chain of blocks: 128 tokens at position 4,000 205 vs 191 us
+// with the block kernel above, 200 at 3,000 192 vs 220) and kAttnTileMin score
+// workgroups (320 tokens at 0: 120 of them, 77 vs 73 us; 384: 168, 79 vs 84).
+constexpr int kAttnTileTokens = 192;
+constexpr int kAttnTileMin = 150;
+constexpr int kWLd = 68;  // LDS row stride of the weights (16 rows on distinct banks)
+
+struct AttnTiles {
+  uint16_t* qn;  // [T][8][4][64]: dim 4i + g of q after norm and RoPE at [g][i]
+  // one record per 16-token tile, head and block
+  float* mb;     // [T / 16][8][max_blocks][16] maxima of the scores
+  float* sb;     // [T / 16][8][max_blocks][16] sums of the weights
+  float* w;      // [T / 16][8][max_blocks][16][4][16] weights: position 4i + g at [g][i]
+};
+
+__global__ __launch_bounds__(640) void attn_qkv_prep_kernel(AttnArgs a, AttnTiles ws) {
+  const int t = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int pos = a.pos0 + t;
+  const bool is_q = wave < kQHeads;
+  const int kvh = wave - kQHeads;
+  const uint16_t* src = is_q ? a.qg + (size_t)t * 4096 + wave * 512 : a.k + (size_t)t * 512 + kvh * kHeadDim;
+  float v[4];
+  load4h(src + 4 * lane, v);
+  head_norm_wave(v, is_q ? a.q_norm_w : a.k_norm_w, lane);
+  rope_wave(v, a.rope + (size_t)pos * 64, lane);
+  if (is_q) {
+    uint16_t* dst = ws.qn + ((size_t)t * kQHeads + wave) * kHeadDim + lane;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) dst[64 * g] = spk::f2h(v[g]);
+  } else {
+    uint16_t* row = a.kv + (size_t)pos * kKvRow + kvh * kHeadDim + 4 * lane;
+    *reinterpret_cast<uint2*>(row) = pack4h(v);
+    *reinterpret_cast<uint2*>(row + 512) =
+        *reinterpret_cast<const uint2*>(a.v + (size_t)t * 512 + kvh * kHeadDim + 4 * lane);
+  }
+}
+
+// Tile z sees blocks 0 .. (z + z0) / 4, z0 = (pos0 + 15) / 16: their number in
+// the tiles before z = m - z0, counted from a tile with z + z0 = 0.
+__host__ __device__ __forceinline__ long long attn_blocks_before(long long m) {
+  const long long q = m / 4, r = m % 4;
+  return 2 * q * (q + 1) + r * (q + 1);
+}
+
+// 1-D grid of the live (tile, block, KV head) triples, the KV head in the low
+// bit: a grid with the blocks past each tile's positions left to exit ran half
+// as fast (workgroups are dealt to the shader engines in turn, and the empty
+// ones fell on the same engines; two blocks per workgroup 2-5% slower).  Wave w
+// = query head 4 kvh + w.  MFMA i contracts dims 4i..4i+3: lane (li, lg)
+// supplies dim 4i + lg of q row li (registers) and of the K row of position
+// 16 (li / 4) + 4 n + li % 4 for chain n (LDS, rows stored [dim % 4][dim / 4],
+// so that a 16-byte read is 8 steps' operands), and ends up with the scores of
+// tokens 4 lg + r at those positions.
+__global__ __launch_bounds__(256, 2) void attn_scores_kernel(AttnArgs a, AttnTiles ws) {
+  __shared__ __align__(16) uint16_t Ks[kAttnBlock][kKLd];
+  const int z0 = (a.pos0 + kAttnRows - 1) / kAttnRows;
+  const int kvh = blockIdx.x & 1;
+  const long long at = (blockIdx.x >> 1) + attn_blocks_before(z0);
+  int tile = 0;
+  for (int step = 1 << 12; step; step >>= 1)  // tiles < 2^13 (positions <= 65536, 16 a tile)
+    if (attn_blocks_before(z0 + tile + step) <= at) tile += step;
+  const int b = (int)(at - attn_blocks_before(z0 + tile));
+  const int t0 = tile * kAttnRows;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int rows = min(kAttnRows, a.tokens - t0);
+  const int npos_max = a.pos0 + t0 + rows;
+  if (kAttnBlock * b >= npos_max) return;  // a part tile may see a block less
+  const int qh = 4 * kvh + wave;
+  const int p0 = 16 * (li >> 2) + (li & 3);  // position of chain 0 in the block; chain n: + 4 n
+  const int p = tid >> 2, q4 = tid & 3;
+  uint4 kr[8];
+  {
+    const int gp = kAttnBlock * b + p;
+    const bool live = gp < npos_max;  // later rows need not be written yet
+    const uint16_t* krow = a.kv + (size_t)(live ? gp : 0) * kKvRow + kvh * kHeadDim + q4 * 64;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      kr[i] = *reinterpret_cast<const uint4*>(krow + 8 * i);
+      if (!live) kr[i] = make_uint4(0, 0, 0, 0);
+    }
+  }
+  uint4 q[8];
+  {
+    const uint16_t* src = ws.qn + ((size_t)(t0 + min(li, rows - 1)) * kQHeads + qh) * kHeadDim + 64 * lg;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = *reinterpret_cast<const uint4*>(src + 8 * i);
+  }
+  {
+    // dims 64 q4 + 8x + (0..7) in kr[x]: dims = g mod 4 of two such pieces are
+    // four consecutive halves of segment g; position 16 h + 4 n + g in row
+    // 16 n + 4 h + g (chain n's lanes)
+    const int row = 16 * ((p >> 2) & 3) + 4 * (p >> 4) + (p & 3);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        uint32_t w[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const uint4& k = kr[4 * h + x];
+          w[x] = __builtin_amdgcn_perm(g < 2 ? k.z : k.w, g < 2 ? k.x : k.y, (g & 1) ? 0x07060302 : 0x05040100);
+        }
+        *reinterpret_cast<uint4*>(&Ks[row][64 * g + 16 * q4 + 8 * h]) = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+  }
+  __syncthreads();
+  const size_t rec = (((size_t)tile * kQHeads + qh) * a.max_blocks + b) * kAttnRows;
+  f32x4 acc[4];
+#pragma unroll
+  for (int n = 0; n < 4; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i8 = 0; i8 < 8; ++i8) {
+    float qf[8], kf[4][8];
+    unpack8(q[i8], qf);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) unpack8(*reinterpret_cast<const uint4*>(&Ks[16 * n + li][64 * lg + 8 * i8]), kf[n]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[e], kf[n][e], acc[n], 0, 0, 0);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = 4 * lg + r;
+    const int seen = row < rows ? a.pos0 + t0 + row - kAttnBlock * b : -1;  // last position of the block it sees
+    float m = -INFINITY, x[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      x[n] = acc[n][r] * 0.0625f;
+      if (p0 + 4 * n <= seen) m = fmaxf(m, x[n]);
+    }
+    m = spk::row_max16(m);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) x[n] = p0 + 4 * n <= seen ? spk::expf_det(x[n] - m) : 0.0f;
+    *reinterpret_cast<float4*>(ws.w + (rec + row) * kAttnBlock + 16 * (li & 3) + 4 * (li >> 2)) =
+        make_float4(x[0], x[1], x[2], x[3]);
+    // the 64-position tree: strides 32 and 16 (h), 8 and 4 (n), 2 and 1 (g)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) x[n] = spk::add_row_shl<4>(spk::add_row_shl<8>(x[n]));
+    const float sum = spk::add_row_shl<1>(spk::add_row_shl<2>((x[0] + x[2]) + (x[1] + x[3])));
+    if (li == 0) {
+      ws.mb[rec + row] = m;
+      ws.sb[rec + row] = sum;
+    }
+  }
+}
+
+// grid (8 x token tiles), the tiles with the most blocks first, the head in
+// the low bits (its V rows stay in one XCD's L2).  Wave w: dims 64w..64w+63 of
+// the tile's 16 rows.  MFMA i contracts positions 4i..4i+3: lane (li, lg)
+// supplies the weight of row li and V's dims 64w + 4 li + n (chain n) of
+// position 4i + lg, and ends up with rows 4 lg + r of those dims.
+// Wavefronts 4..7 stage the next block (V rows, weights, factors) while 0..3
+// run the current one's MFMA, so that the matrix cores do not wait for it.
+__global__ __launch_bounds__(512, 4) void attn_pv_kernel(AttnArgs a, AttnTiles ws) {
+  // V rows, the two 128-byte halves of each 256 swapped in odd rows (the rows
+  // that two 16-lane groups read together then lie on different banks)
+  __shared__ __align__(16) uint16_t Vs[2][kAttnBlock][kHeadDim];
+  __shared__ __align__(16) float Ws[2][kAttnRows][kWLd];  // [row][position % 4][position / 4]
+  __shared__ __align__(16) float Ss[2][kAttnRows], Cs[2][kAttnRows];
+  __shared__ float Ms[kAttnRows];
+  __shared__ int Bad[2][4];
+  const int qh = blockIdx.x & 7, kvh = qh >> 2;
+  const int t0 = ((int)(gridDim.x >> 3) - 1 - (int)(blockIdx.x >> 3)) * kAttnRows;
+  const bool producer = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) != 0;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int rows = min(kAttnRows, a.tokens - t0);
+  const int first = a.pos0 + t0;  // row i sees positions 0 .. first + i
+  const int npos_max = first + rows;
+  const int nb = (npos_max + kAttnBlock - 1) / kAttnBlock;
+  const size_t rec0 = ((size_t)(t0 / kAttnRows) * kQHeads + qh) * a.max_blocks;
+  {
+    const int row = tid >> 4;
+    float m = -INFINITY;
+    if (row < rows)
+      for (int b = tid & 15; kAttnBlock * b <= first + row; b += 16) m = fmaxf(m, ws.mb[(rec0 + b) * kAttnRows + row]);
+    m = spk::row_max16(m);
+    if (producer && (tid & 15) == 0) Ms[row] = m;
+  }
+  __syncthreads();
+  uint4 vr[8];
+  float4 wr;
+  float mr = 0.0f, sr = 0.0f;
+  auto load = [&](int b) {
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const int gp = kAttnBlock * b + (tid >> 5) + 8 * x;
+      vr[x] = *reinterpret_cast<const uint4*>(a.kv + (size_t)(gp < npos_max ? gp : 0) * kKvRow + 512 + kvh * kHeadDim +
+                                              8 * (tid & 31));
+      if (gp >= npos_max) vr[x] = make_uint4(0, 0, 0, 0);
+    }
+    const size_t rec = (rec0 + b) * kAttnRows;
+    wr = *reinterpret_cast<const float4*>(ws.w + rec * kAttnBlock + 4 * tid);
+    mr = ws.mb[rec + li];
+    sr = ws.sb[rec + li];
+  };
+  auto stage = [&](int b, int buf) {
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const int row = (tid >> 5) + 8 * x;
+      *reinterpret_cast<uint4*>(&Vs[buf][row][(8 * (tid & 31)) ^ (64 * (row & 1))]) = vr[x];
+    }
+    if (kAttnBlock * (b + 1) > first + 1) {  // positions that not every row sees: is every V there finite?
+      uint32_t bad = 0;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        const uint32_t v[4] = {vr[x].x, vr[x].y, vr[x].z, vr[x].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          bad |= (v[e] & 0x7c00u) == 0x7c00u;
+          bad |= (v[e] & 0x7c000000u) == 0x7c000000u;
+        }
+      }
+      const int any = __any(bad != 0);
+      if (lane == 0) Bad[buf][wave] = any;
+    }
+    *reinterpret_cast<float4*>(&Ws[buf][tid >> 4][4 * (tid & 15)]) = wr;
+    if (wave == 0) {
+      const float c = spk::expf_det(mr - Ms[li]);  // the rows' combine factors
+      if (lane < kAttnRows) {
+        Cs[buf][lane] = c;
+        Ss[buf][lane] = sr;
+      }
+    }
+  };
+  const int vcol = 64 * wave + 4 * li;
+  f32x4 o[4];
+  float tot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int n = 0; n < 4; ++n) o[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (producer) {
+    load(0);
+    stage(0, 0);
+    if (nb > 1) load(1);
+  }
+  for (int b = 0; b < nb; ++b) {
+    const int buf = b & 1;
+    __syncthreads();
+    if (producer) {
+      if (b + 1 < nb) stage(b + 1, buf ^ 1);
+      if (b + 2 < nb) load(b + 2);
+      continue;
+    }
+    f32x4 acc[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto operands = [&](int i, float (&v)[4]) {
+      const int row = 4 * i + lg;
+      load4h(&Vs[buf][row][vcol ^ (64 * (row & 1))], v);
+    };
+    // All positions, weights past a row's own position zero -- unless one of
+    // the V values that only later rows may see is not finite (0 * inf): then
+    // those positions one at a time, a row past its own keeping its sum.
+    const int nv0 = min(kAttnBlock, max(0, first + 1 - kAttnBlock * b));  // positions every row sees
+    const int nvm = min(kAttnBlock, npos_max - kAttnBlock * b);
+    bool plain = true;
+    if (nv0 < nvm) {
+      const int4 f = *reinterpret_cast<const int4*>(Bad[buf]);
+      plain = (f.x | f.y | f.z | f.w) == 0;
+    }
+    const int quads = plain ? (nvm + 3) >> 2 : nv0 >> 2;
+    auto quad4 = [&](int i4) {  // positions 16 i4 .. 16 i4 + 15
+      const float4 w4 = *reinterpret_cast<const float4*>(&Ws[buf][li][16 * lg + 4 * i4]);
+      const float w[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v[4];
+        operands(4 * i4 + e, v);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], v[n], acc[n], 0, 0, 0);
+      }
+    };
+    if (quads == kAttnBlock / 4) {
+      // straight-line, so that the LDS reads run ahead of the MFMA
+#pragma unroll
+      for (int i4 = 0; i4 < kAttnBlock / 16; ++i4) quad4(i4);
+    } else {
+      int i = 0;
+      for (; i + 4 <= quads; i += 4) quad4(i >> 2);
+      for (; i < quads; ++i) {
+        const float w = Ws[buf][li][16 * lg + i];
+        float v[4];
+        operands(i, v);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, v[n], acc[n], 0, 0, 0);
+      }
+    }
+    if (!plain) {
+      for (int j = nv0 & ~3; j < nvm; ++j) {
+        const bool mine = (j & 3) == lg;
+        const float w = mine ? Ws[buf][li][16 * lg + (j >> 2)] : 0.0f;
+        float v[4];
+        operands(j >> 2, v);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x4f32(w, mine ? v[n] : 0.0f, acc[n], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[n][r] = kAttnBlock * b + j <= first + 4 * lg + r ? d[r] : acc[n][r];
+        }
+      }
+    }
+    const float4 c4 = *reinterpret_cast<const float4*>(&Cs[buf][4 * lg]);
+    const float4 s4 = *reinterpret_cast<const float4*>(&Ss[buf][4 * lg]);
+    const float c[4] = {c4.x, c4.y, c4.z, c4.w}, S[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const bool in = kAttnBlock * b <= first + 4 * lg + r;
+      tot[r] = in ? tot[r] + S[r] * c[r] : tot[r];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) o[n][r] = in ? o[n][r] + acc[n][r] * c[r] : o[n][r];
+    }
+  }
+  if (producer) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = 4 * lg + r;
+    if (row >= rows) continue;
+    const float inv = 1.0f / (tot[r] + 1e-30f);
+    const size_t t = (size_t)(t0 + row);
+    float g[4], y[4];
+    load4h(a.qg + t * 4096 + qh * 512 + 256 + vcol, g);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) y[n] = round16(o[n][r] * inv) * (1.0f / (1.0f + spk::expf_det(-g[n])));
+    *reinterpret_cast<uint2*>(a.out + t * 2048 + qh * kHeadDim + vcol) = pack4h(y);
+  }
+}
+
 // Prefill: K/V rows of positions pos0..pos0+T-1, before any block pass reads
 // them.  grid (T, kv_heads); one wave.
 __global__ __launch_bounds__(64) void attn_store_kv_kernel(AttnArgs a) {
@@ -1626,6 +1984,27 @@ extern "C" int spk_attention_prefill(const SpkAttnArgs* p, int32_t pos0, int32_t
   hipStream_t s = spk::to_hip(stream);
   // Tokens read the K/V rows of earlier tokens of the same call: all rows are
   // stored by one launch before the block passes read them.
+  const int tiles = (tokens + kAttnRows - 1) / kAttnRows;
+  const int z0 = (pos0 + kAttnRows - 1) / kAttnRows;
+  const long long score_wgs = kKvHeads * (attn_blocks_before((long long)z0 + tiles) - attn_blocks_before(z0));
+  if (tokens >= kAttnTileTokens && score_wgs >= kAttnTileMin) {
+    // 4,096 + 2,112 max_blocks bytes per token (rounded up to whole tiles) of
+    // the partials' 8,256 max_blocks
+    const size_t recs = (size_t)tiles * kAttnRows * kQHeads * a.max_blocks;
+    AttnTiles w;
+    w.qn = static_cast<uint16_t*>(p->workspace);
+    w.mb = reinterpret_cast<float*>(w.qn + (size_t)tokens * kQHeads * kHeadDim);
+    w.sb = w.mb + recs;
+    w.w = w.sb + recs;
+    hipLaunchKernelGGL(attn_qkv_prep_kernel, dim3(tokens), dim3(640), 0, s, a, w);
+    rc = spk::check_launch("spk_attention_prefill (store)");
+    if (rc) return rc;
+    hipLaunchKernelGGL(attn_scores_kernel, dim3((unsigned)score_wgs), dim3(256), 0, s, a, w);
+    rc = spk::check_launch("spk_attention_prefill (scores)");
+    if (rc) return rc;
+    hipLaunchKernelGGL(attn_pv_kernel, dim3(kQHeads * tiles), dim3(512), 0, s, a, w);
+    return spk::check_launch("spk_attention_prefill (values)");
+  }
   hipLaunchKernelGGL(attn_store_kv_kernel, dim3(tokens, kKvHeads), dim3(64), 0, s, a);
   rc = spk::check_launch("spk_attention_prefill (store)");
   if (rc) return rc;

@@ -340,6 +340,32 @@ def test_attention_prefill_bitexact(dev, pos0, T):
     assert np.array_equal(_u16(d["out"]), exp)
 
 
+# the matrix-core tiles (192 tokens and 150 score workgroups up): whole and part
+# tiles, starts on and off tile and block edges, a block seen by part of a tile
+@pytest.mark.parametrize("pos0,T", [(0, 385), (0, 400), (61, 335), (190, 256), (48, 337), (300, 192), (305, 199)])
+def test_attention_prefill_tiles_bitexact(dev, pos0, T):
+    """The matrix-core path against the oracle, bit for bit; then the same with
+    one value of V infinite: rows that may not see it are unchanged."""
+    from spock_amd import _lib
+    print(f"[attention prefill tiles pos0={pos0} T={T}]", flush=True)
+    max_seq = 640
+    rope, kv, qg, k, v, qn, kn = _attn_inputs(300 + T, max_seq, pos0, T)
+    kv[(pos0 + T) * 1024:] = 0x7E00  # rows past the prompt (NaN) are not read
+    for inf_at in (None, T - 9):
+        if inf_at is not None:
+            v = v.copy()
+            v[inf_at * 512 + 300] = 0x7C00
+        a, d = _attn_args(dev, rope, kv, qg, k, v, qn, kn, max_seq, T, pos0 + T)
+        _lib.check(_lib.lib().spk_attention_prefill(C.byref(a), pos0, T, _stream()), "spk_attention_prefill")
+        torch.cuda.synchronize()
+        exp, ekv = _oracle_attention(rope, kv, qg, k, v, qn, kn, pos0, T)
+        assert np.array_equal(_u16(d["kv"]), ekv)
+        got, exp = _u16(d["out"]).view(np.float16), exp.view(np.float16)
+        assert np.array_equal(np.isnan(got), np.isnan(exp))
+        ok = ~np.isnan(exp)
+        assert np.array_equal(got[ok].view(np.uint16), exp[ok].view(np.uint16))
+
+
 def test_attention_decode_position_out_of_range_writes_nothing(dev):
     from spock_amd import _lib
     max_seq = 128
