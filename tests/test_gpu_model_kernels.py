@@ -415,6 +415,23 @@ def test_elementwise_gates_bitexact(dev):
     assert np.array_equal(_u16(y2), e2)
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 4097])
+@pytest.mark.parametrize("shift", [0, 1])  # 16-byte aligned rows, and not
+def test_silu_gate_in_place_any_length_and_alignment(dev, n, shift):
+    from spock_amd import _lib
+    g, u = _rand16(43, n, 3.0), _rand16(44, n)
+    dg, du = torch.zeros(n + 9, dtype=torch.float16, device=dev), _h(u, dev)
+    dg[shift:shift + n] = _h(g, dev)
+    _lib.check(_lib.lib().spk_silu_gate_f16(dg.data_ptr() + 2 * shift, du.data_ptr(), dg.data_ptr() + 2 * shift, n,
+                                            _stream()), "silu")
+    torch.cuda.synchronize()
+    want = np.zeros(n, np.uint16)
+    _om().orc_silu_gate(_p(g), _p(u), _p(want), n)
+    got = _u16(dg)
+    assert np.array_equal(got[shift:shift + n], want)
+    assert not got[:shift].any() and not got[shift + n:].any()
+
+
 def test_embedding_rows(dev):
     from spock_amd import _lib
     V = 300
@@ -430,7 +447,7 @@ def test_embedding_rows(dev):
         assert np.array_equal(got[i], E[t] if 0 <= t < V else np.zeros(1024, np.uint16))
 
 
-@pytest.mark.parametrize("T", [1, 5, 64, 133])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 8, 64, 133])  # runs of 4 tokens per wave
 def test_deltanet_prefill_conv_bitexact(dev, oracle, T):
     from spock_amd import _lib
     print(f"[dn prefill conv T={T}]", flush=True)
