@@ -1,6 +1,4 @@
-// chunk.hip -- gated-DeltaNet chunk prefill (WY/UT chunk rule) on the matrix
-// cores: fp32 MFMA, and for fp16 inputs the f16 MFMA with the fp32 operands of
-// the state scan held as pairs of halves.
+// chunk.hip -- gated-DeltaNet chunk prefill (WY/UT chunk rule) on fp32 MFMA.
 //
 // Math (deltanet_chunk.cpp:134-268, deltanet_chunk_prefill_tiled.comp:116-262):
 // per (sequence, head) and chunk of C=64 tokens with cumulative log-decay
@@ -30,15 +28,13 @@
 //     and K' are MFMA products over the nonzero blocks of T with Ks applied to
 //     the K operand as it is read.  They go to the workspace with the
 //     per-token scales.
-//  2. the state scan -- one workgroup per (sequence, head, column tile of the
-//     value dim): columns of S evolve independently, so the sequential chunk
-//     scan runs on up to 8*H*num_seqs workgroups.  Wavefront M owns token block
-//     M of K S, Q S, R and the output, and state rows 32M..32M+31 of the
-//     update (S += K'^T R), with the next chunk's operands prefetched into
-//     registers during the current one.  fp32 inputs: chunk_state_kernel, all
-//     16x16x4 fp32 MFMA, state tile in LDS.  fp16 inputs:
-//     chunk_scan_split_kernel, 16x16x32 f16 MFMA on split operands, state in
-//     registers.
+//  2. chunk_state_kernel -- one workgroup per (sequence, head, 16-column tile
+//     of the value dim): columns of S evolve independently, so the sequential
+//     chunk scan runs on 8*H*num_seqs workgroups.  The 128x16 state tile lives
+//     in LDS; wavefront M owns token block M of K S, Q S, R and the output,
+//     and state rows 32M..32M+31 of the update (S += K'^T R), all 16x16x4
+//     MFMA, with the next chunk's operands prefetched into registers during
+//     the current one.
 // MFMA operand trick: the contraction index of a 16x16x4 step is a free
 // permutation, so lane (m = l%16, g = l/16) reads a float4 at k = 16u + 4g and
 // feeds its elements to 4 consecutive steps; the B operand uses the same map.
@@ -95,13 +91,6 @@ constexpr int kWsQs = 12288;
 constexpr int kWsC1 = 12352;
 constexpr int kWsC2 = 12416;
 constexpr int kWsMisc = 12480;
-// fp16 inputs: K' and A T as split halves (see pow2_for), in the scan's
-// 16x16x32 fragment order; 8 halves per lane of a 32-token pair P of blocks:
-// tokens 32P+4lg+e (e < 4) and 32P+16+4lg+e.
-//   K'  [M 4][t 2][P 2][hi, lo][lane][8]   key dim 32M+8(li/4)+4t+li%4
-//   AT  [M 4][P <= M/2][hi, lo][lane][8]   row 16M+li (fragments from kAtFrag[M])
-//   Misc[M 4][e^{gL}, inverse scale of K' tile (M, 0), (M, 1), of A T's rows M]
-constexpr int kAtFrag[4] = {0, 2, 4, 8};
 constexpr int kWsStride = 12544;  // 50176 bytes, a multiple of 256
 // Word 3 of a raw buffer resource on gfx9-family parts: 32-bit data format,
 // which untyped loads/stores need for the num_records range check to apply.
@@ -224,17 +213,25 @@ template <> struct RawOf<uint16_t> {
     return make_float4(spk::h2f((uint16_t)(x & 0xffffu)), spk::h2f((uint16_t)(x >> 16)),
                        spk::h2f((uint16_t)(y & 0xffffu)), spk::h2f((uint16_t)(y >> 16)));
   }
+  // 8 consecutive halves (one 16-byte load), half i converted at use
+  typedef uint4 R8;
+  static __device__ __forceinline__ R8 ld8(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+  static __device__ __forceinline__ float get8(const R8& r, int i) {
+    const uint32_t w = (i >> 1) == 0 ? r.x : (i >> 1) == 1 ? r.y : (i >> 1) == 2 ? r.z : r.w;
+    return spk::h2f((uint16_t)((i & 1) ? w >> 16 : w & 0xffffu));
+  }
 };
 
-// V elements of the fp32 scan's stage B: row 16M+li, value columns n0+4lg..+3
-// (one 16-byte load per lane), read through a buffer resource of the chunk's
-// len rows, so rows past the chunk read 0 (the hardware range check) with no
-// clamp or select.
+// V elements of the scan's stage B: row 16M+li, value columns n0+4lg..+3 (one
+// 8-byte (fp16) or 16-byte (fp32) load per lane), read through a buffer
+// resource of the chunk's len rows, so rows past the chunk read 0 (the
+// hardware range check) with no clamp or select.
 // The whole byte offset goes in the VGPR offset and the scalar offset stays 0:
 // on gfx9-family raw buffers the range check compares only voffset +
 // inst_offset with num_records, so a row offset passed as soffset would read
 // past the chunk (the next sequence's rows, or past the tensor) unchecked.
-struct VTile {
+template <typename TIn> struct VTile;
+template <> struct VTile<float> {
   float x[4];
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int voff) {
     const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0);
@@ -242,6 +239,17 @@ struct VTile {
     for (int e = 0; e < 4; ++e) x[e] = __uint_as_float(v[e]);
   }
   __device__ __forceinline__ float get(int e) const { return x[e]; }
+};
+template <> struct VTile<uint16_t> {
+  uint32_t x[2];
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int voff) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0);
+    x[0] = v[0];
+    x[1] = v[1];
+  }
+  __device__ __forceinline__ float get(int e) const {
+    return spk::h2f((uint16_t)((e & 1) ? x[e / 2] >> 16 : x[e / 2] & 0xffffu));
+  }
 };
 
 // K rows staged in LDS in the input type (fp16 rows stay fp16) with a
@@ -333,83 +341,7 @@ __host__ __device__ constexpr int gram_nj() {  // K row blocks read: 0 .. nJ-1
 }
 
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ f4v mfma32h(const u32x4v& a, const u32x4v& b, f4v c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8v, a), __builtin_bit_cast(h8v, b), c, 0, 0, 0);
-}
-
-// fp32 operands on the f16 matrix cores (fp16 inputs' path): x is held as
-// hi + lo, two halves of x times a power of two that brings the largest |x|
-// of its group into [2^14, 2^15).  hi is x rounded to 11 bits, lo the rest
-// rounded to 11 bits, so hi + lo keeps 23 bits of every element down to 2^-17
-// of the group's largest (fp32 keeps 24) and an absolute 2^-39 of the largest
-// below that.  A product of two such operands is hi.hi + hi.lo + lo.hi (the
-// dropped lo.lo is below 2^-23 of the product), each product of halves exact in
-// fp32 and accumulated in fp32; a product with raw fp16 inputs needs two.
-struct Pow2 {
-  float s, inv;
-};
-// m: the group's largest |x| (NaN ignored by the caller's maxima).  The
-// scales' exponents are clamped so that both are normal numbers; an infinite
-// maximum gives 2^-114 and the group's finite elements vanish beside it.
-__device__ __forceinline__ Pow2 pow2_for(float m) {
-  const int e = (int)((__float_as_uint(m) >> 23) & 0xffu);
-  const int sb = min(268 - e, 253);
-  return Pow2{__uint_as_float((uint32_t)sb << 23), __uint_as_float((uint32_t)(254 - sb) << 23)};
-}
-// Two elements -> one word of hi halves and one of lo halves (v_fma_mix*_f16:
-// the exact remainder a - hi rounded once).
-__device__ __forceinline__ void split2(float x, float y, float s, uint32_t& hi, uint32_t& lo) {
-  const float a = x * s, b = y * s;
-  const h2v h = {(_Float16)a, (_Float16)b};
-  hi = __builtin_bit_cast(uint32_t, h);
-  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(a));
-  asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(b));
-}
-__device__ __forceinline__ void split8(const f4v& x, const f4v& y, float s, u32x4v& hi, u32x4v& lo) {
-  uint32_t h[4], l[4];
-  split2(x[0], x[1], s, h[0], l[0]);
-  split2(x[2], x[3], s, h[1], l[1]);
-  split2(y[0], y[1], s, h[2], l[2]);
-  split2(y[2], y[3], s, h[3], l[3]);
-  hi = u32x4v{h[0], h[1], h[2], h[3]};
-  lo = u32x4v{l[0], l[1], l[2], l[3]};
-}
-__device__ __forceinline__ float absmax4(const f4v& x, float m) {
-  m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), m);
-  return fmaxf(fmaxf(fabsf(x[2]), fabsf(x[3])), m);
-}
-// Maximum over the four lanes of equal li of a non-negative float's bits.
-__device__ __forceinline__ uint32_t col_max(uint32_t m) {
-  const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
-  m = max(r[0], r[1]);
-  const auto q = __builtin_amdgcn_permlane32_swap(m, m, false, false);
-  return max(q[0], q[1]);
-}
-// The largest finite |x| of N values per lane over the four lanes of equal li
-// (bits).  An infinity or NaN leaves the plain maximum not finite; only then
-// the values are looked at one by one.
-template <int N>
-__device__ __forceinline__ uint32_t col_absmax(const f4v (&x)[N]) {
-  float f = 0.0f;
-#pragma unroll
-  for (int i = 0; i < N; ++i) f = absmax4(x[i], f);
-  const uint32_t m = col_max(__float_as_uint(f));
-  if (__builtin_expect(__any(m >= 0x7f800000u), 0)) {
-    uint32_t u = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t w = __float_as_uint(x[i][r]) & 0x7fffffffu;
-        u = max(u, w < 0x7f800000u ? w : 0u);
-      }
-    return col_max(u);
-  }
-  return m;
-}
 
 template <typename TIn, unsigned KMASK, int QB>
 __device__ __forceinline__ void gram_tiles(const typename RowStage<TIn>::T* sK, const float4 (&qa)[8],
@@ -530,39 +462,6 @@ __device__ __forceinline__ void at_store(const f4v (&acc)[5], const float* sL, c
   }
 }
 
-// The same as split halves, one scale per row block QB.
-template <unsigned KMASK, int QB>
-__device__ __forceinline__ void at_store_split(const f4v (&acc)[5], const float* sL, const float* sT, float* ws,
-                                               int li, int lg, int lane) {
-  if constexpr (QB >= 0) {
-    constexpr int nK = gram_ntiles<KMASK, -1>();
-    f4v x[4];
-    float m = 0.0f;
-#pragma unroll
-    for (int K = 0; K < 4; ++K) x[K] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int K = 0; K <= QB; ++K) {
-#pragma unroll
-      for (int J = K; J <= QB; ++J) {
-        const float* tb = tblk(sL, sT, J, K);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[K] = mfma4(tb[(4 * lg + e) * 16 + li], acc[nK + J][e], x[K]);
-      }
-      m = absmax4(x[K], m);
-    }
-    const Pow2 sc = pow2_for(spk::wave_max(m));
-#pragma unroll
-    for (int P = 0; P <= QB / 2; ++P) {
-      u32x4v hi, lo;
-      split8(x[2 * P], x[2 * P + 1], sc.s, hi, lo);
-      float* d = ws + kWsA + (kAtFrag[QB] + 2 * P) * 256 + lane * 4;
-      __builtin_nontemporal_store(hi, reinterpret_cast<u32x4v*>(d));
-      __builtin_nontemporal_store(lo, reinterpret_cast<u32x4v*>(d + 256));
-    }
-    if (lane == 0) ws[kWsMisc + 4 * QB + 3] = sc.inv;
-  }
-}
-
 // Gram work of wavefront `wave` in part `part` of PARTS, dispatched to the
 // instance (KMASK, QB) that holds it.  Without a split: row block 3-w and
 // query block w (five tiles).  With one, only the wavefronts that own their
@@ -595,7 +494,6 @@ struct GramStoreOp {
     gram_store<KM, QB>(acc, sG, sB, sIK, iq_scale, sL, li, lg);
   }
 };
-template <bool SPLIT>
 struct AtStoreOp {
   const f4v (&acc)[5];
   const float *sL, *sT;
@@ -603,10 +501,7 @@ struct AtStoreOp {
   int li, lg, lane;
   template <unsigned KM, int QB>
   __device__ __forceinline__ void run() const {
-    if constexpr (SPLIT)
-      at_store_split<KM, QB>(acc, sL, sT, ws, li, lg, lane);
-    else
-      at_store<KM, QB>(acc, sL, sT, ws, li, lg, lane);
+    at_store<KM, QB>(acc, sL, sT, ws, li, lg, lane);
   }
 };
 
@@ -678,7 +573,6 @@ template <typename TIn, int PARTS>
 __global__ __launch_bounds__(256, sizeof(TIn) == 2 ? 5 : 1) void chunk_intra_kernel(ChunkParams p) {
   typedef RawOf<TIn> R;
   typedef RowStage<TIn> RS;
-  constexpr bool kSplit = std::is_same<TIn, uint16_t>::value;  // record of split halves
   __shared__ __align__(16) typename RS::T sK[64 * RS::kLd];  // K rows, raw
   __shared__ __align__(16) float sL[10 * 256];  // L blocks; diagonal blocks become T's
   __shared__ __align__(16) float sT[3 * 256];   // T_21, T_31, T_32
@@ -815,7 +709,7 @@ __global__ __launch_bounds__(256, sizeof(TIn) == 2 ? 5 : 1) void chunk_intra_ker
       ws[kWsC2 + tid] = sB[tid] * expf(sG[tid]) * sIK[tid];
     }
   }
-  if (tid < (kSplit ? 4 : 1) && part == 0) ws[kWsMisc + 4 * tid] = expf(gL);
+  if (tid == 0 && part == 0) ws[kWsMisc] = expf(gL);
   __syncthreads();
 
   // ---- diagonal blocks of T by forward substitution, lane j < 16 of wave w
@@ -863,7 +757,7 @@ __global__ __launch_bounds__(256, sizeof(TIn) == 2 ? 5 : 1) void chunk_intra_ker
   }
 
   // ---- A T for this wavefront's A block (the owner of query block `wave`)
-  gram_dispatch<PARTS>(part, wave, AtStoreOp<kSplit>{acc, sL, sT, ws, li, lg, lane});
+  gram_dispatch<PARTS>(part, wave, AtStoreOp{acc, sL, sT, ws, li, lg, lane});
 
   // ---- K' = T^T diag(Ks) K, by 16-column key tiles ct = 2M + t (keys
   // 32M + 2c + t, c = 0..15: the pair of adjacent keys a lane of the scan's
@@ -880,7 +774,7 @@ __global__ __launch_bounds__(256, sizeof(TIn) == 2 ? 5 : 1) void chunk_intra_ker
     const bool odd_rows = (wave >> 1) != 0;
     const unsigned umask = PARTS == 8 ? (1u << wave) : PARTS == 4 ? (odd_rows ? 0x6u : 0x9u) : 0xFu;
     const int jmin = PARTS == 8 ? wave : PARTS == 4 ? (odd_rows ? 1 : 0) : 0;
-    const int n = kSplit ? 32 * M + 8 * (li >> 2) + 4 * t + (li & 3) : 32 * M + 2 * li + t;
+    const int n = 32 * M + 2 * li + t;
     f4v ak[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) ak[u] = f4v{0.f, 0.f, 0.f, 0.f};
@@ -900,45 +794,10 @@ __global__ __launch_bounds__(256, sizeof(TIn) == 2 ? 5 : 1) void chunk_intra_ker
         for (int e = 0; e < 4; ++e) ak[u] = mfma4(tb[(4 * lg + e) * 16 + li], kb[e], ak[u]);
       }
     }
-    if constexpr (kSplit) {
-      // one scale per tile (M, t) over all 64 tokens: with 4 or 8 parts the
-      // wavefronts that share the tile exchange their maxima
-      float m = 0.0f;
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if ((umask >> u) & 1u) m = absmax4(ak[u], m);
-      m = spk::wave_max(m);
-      if constexpr (PARTS >= 4) {
-        if (lane == 0) sG[wave] = m;  // gcum is no longer read
-        __syncthreads();
-        m = PARTS == 4 ? fmaxf(sG[wave & 1], sG[2 + (wave & 1)]) : fmaxf(fmaxf(sG[0], sG[1]), fmaxf(sG[2], sG[3]));
-      }
-      const Pow2 sc = pow2_for(m);
-      float* d = ws + kWsKp + (M * 2 + t) * 1024 + lane * 4;
-#pragma unroll
-      for (int P = 0; P < 2; ++P) {
-        u32x4v hi, lo;
-        split8(ak[2 * P], ak[2 * P + 1], sc.s, hi, lo);
-        float* dh = d + P * 512;
-        if constexpr (PARTS < 4) {
-          __builtin_nontemporal_store(hi, reinterpret_cast<u32x4v*>(dh));
-          __builtin_nontemporal_store(lo, reinterpret_cast<u32x4v*>(dh + 256));
-        } else {
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-            if ((umask >> (2 * P + b)) & 1u) {
-              ws_store(dh + 2 * b, hi[2 * b], hi[2 * b + 1]);
-              ws_store(dh + 256 + 2 * b, lo[2 * b], lo[2 * b + 1]);
-            }
-        }
-      }
-      if (lane == 0) ws[kWsMisc + 4 * M + 1 + t] = sc.inv;
-    } else {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        if (!((umask >> u) & 1u)) continue;
-        ws_store(ws + kWsKp + (((M * 4 + u) * 2 + t) * 64 + lane) * 4, ak[u][0], ak[u][1], ak[u][2], ak[u][3]);
-      }
+    for (int u = 0; u < 4; ++u) {
+      if (!((umask >> u) & 1u)) continue;
+      ws_store(ws + kWsKp + (((M * 4 + u) * 2 + t) * 64 + lane) * 4, ak[u][0], ak[u][1], ak[u][2], ak[u][3]);
     }
     __builtin_amdgcn_sched_barrier(0);  // one column tile's operands live at a time
   }
@@ -966,12 +825,14 @@ constexpr int kLdVT = 68;   // LDS row stride of the transposed R tile (floats)
 
 // Operands of one chunk for stage A (prefetched a chunk ahead) and for stages
 // B-D (loaded at the start of the chunk's own step, in flight during stage A).
+template <typename TIn>
 struct ScanEarly {
-  RawOf<float>::R8 k[4];  // raw K rows: token 16M+li, key dims 32j+8lg..+7
-  RawOf<float>::R8 q[4];  // raw Q rows, same map
+  typename RawOf<TIn>::R8 k[4];  // raw K rows: token 16M+li, key dims 32j+8lg..+7
+  typename RawOf<TIn>::R8 q[4];  // raw Q rows, same map
 };
+template <typename TIn>
 struct ScanLate {
-  VTile v;  // V: token 16M+li, columns n0+4lg..+3
+  VTile<TIn> v;  // V: token 16M+li, columns n0+4lg..+3
   float c1;      // beta of token 16M+li
   float c2;      // beta e^gcum ik of the same token
   float qs;      // Qs of the same token
@@ -980,21 +841,27 @@ struct ScanLate {
   float4 kq[4][2];  // K'[16u+4lg..+3][32M+2li+t] at [u][t]
 };
 
-// Sequential chunk scan over one 128x16 state tile, fp32 inputs: one workgroup
-// of 4 wavefronts per (sequence, head, 16-column tile).  Wavefront M:
+// Sequential chunk scan over one 128x16 state tile: one workgroup of 4
+// wavefronts per (sequence, head, 16-column tile), so a 16-head batch of 8
+// sequences gives 1024 workgroups and three run on each CU (independent
+// barriers: one workgroup's waits are the others' issue slots).  Wavefront M:
 //   A  rows of token block M: K_M S and Q_M S
 //   B  R = beta V - (beta e^g ik) (K S)  -> LDS
 //   C  o = qs (Q S) + (A T) R -> core
 //   D  S rows 32M..32M+31 <- e^{gL} S + K'^T R
-// 100-112 MFMA per wavefront per chunk (stage C: 4 (M+1)).  Two workgroups per
-// CU: at 168 VGPRs (three) the fp32 operands spilled 236 bytes per lane inside
-// the chunk loop.
+// 100-112 MFMA per wavefront per chunk (stage C: 4 (M+1)).
+// MINB workgroups per CU.  fp16 inputs, large launches: three (168 VGPRs;
+// the instance spills 16 bytes per lane): more resident wavefronts measured faster than two
+// workgroups holding both operand sets double-buffered.  fp32 inputs hold
+// twice the Q and K operand registers: at 168 VGPRs they spilled 236 bytes
+// per lane inside the chunk loop (6.5-9 us per chunk step against 3.1 for
+// fp16), so they run two workgroups per CU without spilling, as do small
+// fp16 launches.
 // ZERO_INIT (no initial state): S is zero entering each sequence's first
 // chunk, so that chunk's K S and Q S are exactly zero and stage A is skipped.
-template <bool ZERO_INIT>
-__global__ __launch_bounds__(256, 2) void chunk_state_kernel(ChunkParams p) {
-  typedef float TIn;
-  typedef RawOf<float> R;
+template <typename TIn, bool ZERO_INIT, int MINB>
+__global__ __launch_bounds__(256, MINB) void chunk_state_kernel(ChunkParams p) {
+  typedef RawOf<TIn> R;
   // S tile and R stored transposed ([column][contraction index]) so one
   // ds_read_b128 feeds four consecutive MFMA steps; strides 132 and 68 keep
   // the 8-lane groups of a b128 access on distinct banks.
@@ -1063,7 +930,7 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(ChunkParams p) {
   const size_t in_off = ((size_t)h * p.N + t_begin) * kD;
   const TIn* qin = static_cast<const TIn*>(p.q) + in_off + 8 * lg;
   const TIn* kin = static_cast<const TIn*>(p.k) + in_off + 8 * lg;
-  auto load_early = [&](ScanEarly& e, int c) {
+  auto load_early = [&](ScanEarly<TIn>& e, int c) {
     const int row = 16 * M + li;
     const size_t ro = (size_t)(c * kC + (row < L - c * kC ? row : 0)) * kD;
 #pragma unroll
@@ -1076,7 +943,7 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(ChunkParams p) {
   // complete in issue order): V through a buffer resource of the chunk's len
   // rows (padding rows read 0) and the per-token factors, then A T, then K'.
   const TIn* vin = static_cast<const TIn*>(p.v) + in_off;
-  auto load_late = [&](ScanLate& l, int c) {
+  auto load_late = [&](ScanLate<TIn>& l, int c) {
     const float* ws = record(c);
     const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<TIn*>(vin + (size_t)c * kC * kD), 0, min(kC, L - c * kC) * kD * (int)sizeof(TIn), kBufDword3);
@@ -1096,7 +963,7 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(ChunkParams p) {
   };
 
   // zero_s: S is zero (first chunk without an initial state)
-  auto step = [&](const ScanEarly& e, const ScanLate& l, int c, auto zero_s) {
+  auto step = [&](const ScanEarly<TIn>& e, const ScanLate<TIn>& l, int c, auto zero_s) {
     const int tok0 = t_begin + c * kC;
     const int len = min(kC, L - c * kC);
 
@@ -1218,8 +1085,8 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(ChunkParams p) {
   // first chunk to drop its stage A at compile time (a run-time flag, or the
   // peeled loop for every launch, made the fp16 instance spill more).
   using NZ = std::integral_constant<bool, false>;
-  ScanEarly ea, eb;
-  ScanLate lt;
+  ScanEarly<TIn> ea, eb;
+  ScanLate<TIn> lt;
   if constexpr (ZERO_INIT) {
     __syncthreads();
     if (nchunks > 0) {
@@ -1256,364 +1123,6 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(ChunkParams p) {
     const int c = i & 15;
     outs[r * kD + n0 + c] = sST[c * kLdST + r];
   }
-}
-
-// ---- the scan for fp16 inputs ----------------------------------------------
-// The same steps as chunk_state_kernel, with every fp32 operand (S, R, K', A T)
-// as split halves on the 16x16x32 f16 MFMA: 16 cycles for 32 contraction
-// elements where the fp32 form takes 8 x 32, so a chunk step of a 16-column
-// tile issues 31-34 MFMA of 16 cycles per wavefront instead of 100-112 of 32.
-// The fp32 form was bound by that issue (68% of the scan; 8 ragged sequences,
-// 34,878 tokens, 16 heads: 588 us of a 723 us call); this one is bound by the
-// chain of a chunk step (four barriers, the column maxima, VALU work on the
-// halves) and, with two workgroups per CU, by its loads: the same call 494 us,
-// 370 with the loads left out; one 2048-token sequence 104 -> 74 us.
-//
-// A wavefront holds S[32M+8lg+4t+r][column] in registers as the D fragments of
-// tiles t = 0, 1, whose rows are ordered so that the lane's eight elements are
-// exactly its B-operand fragment for dims 32M..32M+31: the update needs no
-// transpose, and stage A's operands pass through LDS as written.  R likewise:
-// a D fragment of token block 2P and one of 2P+1 are the B operand of pair P.
-// Scales (pow2_for) are per value column, common to the four wavefronts: each
-// publishes its column maximum, and after a barrier all form the same scale.
-// Columns never share one, so a column's range or a non-finite value stays its
-// own; a finite R element keeps 2^-39 of its column's largest in the chunk.
-// NT: 16-column tiles per workgroup (columns col, col+NT.. interleaved); every
-// column's arithmetic is the same for either.
-template <int NT, int MINB>
-__global__ __launch_bounds__(256, MINB) void chunk_scan_split_kernel(ChunkParams p) {
-  constexpr int kT = 8 / NT;  // column tiles per (sequence, head)
-  typedef typename std::conditional<NT == 1, u32x2v, u32x4v>::type VRow;
-  // S and R as split halves in MFMA operand order (B operand: lane (li, lg)
-  // holds 8 contraction elements of column li), one scale per column, from
-  // the four wavefronts' column maxima
-  __shared__ u32x4v sS[NT][4][2][64];
-  __shared__ u32x4v sR[NT][2][2][64];
-  __shared__ uint32_t sSm[NT][16][4];
-  __shared__ uint32_t sRm[NT][16][4];
-  // a wavefront's own V rows (16 tokens x 16 NT columns) and factors (16 each
-  // of c1, c2, Qs, then e^{gL} and the inverse scales of K' and A T)
-  __shared__ VRow sV[4][64];
-  __shared__ f4v sFac[4][16];
-
-  const int b = blockIdx.x;
-  const int groups = (p.nsel > 0 ? p.nsel : p.S) * p.H;
-  int gi, tile;
-  if ((groups & 7) == 0) {
-    gi = (b / (8 * kT)) * 8 + (b & 7);
-    tile = (b >> 3) % kT;
-  } else {
-    gi = b / kT;
-    tile = b % kT;
-  }
-  const int h = gi % p.H;
-  const int slot = gi / p.H;
-  const int seq = p.nsel > 0 ? p.sel_seq[slot] : lpt_sequence(p, slot);
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int M = __builtin_amdgcn_readfirstlane(((tid >> 6) + b) & 3);
-  const int li = lane & 15;
-  const int lg = lane >> 4;
-  const int n0 = tile * 16 * NT;
-  const int col = n0 + NT * li;  // first value column of the lane
-
-  int t_begin = 0, L = p.N, co = 0;
-  if (p.nsel > 0) {
-    t_begin = p.sel_t0[slot];
-    L = p.sel_len[slot];
-    co = p.sel_co[slot];
-  } else if (p.cu) {
-    L = seq_span(p, seq, t_begin);
-    for (int s = 0; s < seq; ++s) {
-      int ts;
-      co += (seq_span(p, s, ts) + kC - 1) / kC;
-    }
-    if (co + (L + kC - 1) / kC > p.chunks) L = 0;
-  }
-  const int nchunks = (L + kC - 1) / kC;
-
-  const size_t in_off = ((size_t)h * p.N + t_begin) * kD;
-  const uint16_t* qin = static_cast<const uint16_t*>(p.q) + in_off + 8 * lg;
-  const uint16_t* kin = static_cast<const uint16_t*>(p.k) + in_off + 8 * lg;
-  const uint16_t* vin = static_cast<const uint16_t*>(p.v) + in_off;
-  auto record = [&](int c) { return p.ws + ((size_t)(co + c) * p.H + h) * kWsStride; };
-  // Operands of one chunk, each loaded again for the next chunk as soon as
-  // the current one has used it
-  u32x4v k[4], q[4], kp[2][2][2], at[2][2];
-  VRow v;
-  f4v fac;
-  auto row_off = [&](int c) {
-    const int row = 16 * M + li;
-    return (size_t)(c * kC + (row < L - c * kC ? row : 0)) * kD;
-  };
-  auto load_k = [&](int c) {
-    const size_t ro = row_off(c);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) k[j] = *reinterpret_cast<const u32x4v*>(kin + ro + 32 * j);
-  };
-  auto load_q = [&](int c) {
-    const size_t ro = row_off(c);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) q[j] = *reinterpret_cast<const u32x4v*>(qin + ro + 32 * j);
-  };
-  // lanes 0-3: c1, 4-7: c2, 8-11: Qs of tokens 16M.. (4 each), 12: Misc[M]
-  const int fac_at = lane < 12 ? (lane < 4 ? kWsC1 : lane < 8 ? kWsC2 : kWsQs) + 16 * M + 4 * (lane & 3) : kWsMisc + 4 * M;
-  auto load_v = [&](int c) {
-    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(vin + (size_t)c * kC * kD), 0, min(kC, L - c * kC) * kD * 2, kBufDword3);
-    const int off = ((16 * M + (lane >> 2)) * kD + n0 + 4 * NT * (lane & 3)) * 2;
-    if constexpr (NT == 1)
-      v = __builtin_bit_cast(VRow, __builtin_amdgcn_raw_buffer_load_b64(vr, off, 0, 0));
-    else
-      v = __builtin_bit_cast(VRow, __builtin_amdgcn_raw_buffer_load_b128(vr, off, 0, 0));
-    fac = *reinterpret_cast<const f4v*>(record(c) + fac_at);
-  };
-  auto load_kp = [&](int c, int t) {
-    const float* ws = record(c) + kWsKp + M * 2048 + lane * 4;
-#pragma unroll
-    for (int P = 0; P < 2; ++P)
-#pragma unroll
-      for (int x = 0; x < 2; ++x) kp[t][P][x] = *reinterpret_cast<const u32x4v*>(ws + ((t * 2 + P) * 2 + x) * 256);
-  };
-  const int at_off = kWsA + (M < 2 ? 2 * M : 4 * M - 4) * 256 + lane * 4;
-  auto load_at = [&](int c) {
-    const float* ws = record(c) + at_off;
-#pragma unroll
-    for (int P = 0; P < 2; ++P)
-#pragma unroll
-      for (int x = 0; x < 2; ++x) at[P][x] = *reinterpret_cast<const u32x4v*>(ws + ((M >= 2 ? 2 * P : 0) + x) * 256);
-  };
-
-  // The state in registers: s[nt][t][r] = S[32M+8lg+4t+r][col+nt]
-  f4v s[NT][2];
-  const size_t st_off = ((size_t)seq * p.H + h) * kD * kD + (size_t)(32 * M + 8 * lg) * kD + col;
-  if (p.init) {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[nt][t][r] = p.init[st_off + (4 * t + r) * kD + nt];
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) s[nt][0] = s[nt][1] = f4v{0.f, 0.f, 0.f, 0.f};
-  }
-  float sinv[NT];  // inverse scale of the state column, the same in every wavefront
-  auto publish = [&](uint32_t (&dst)[16][4], uint32_t m) {
-    if (lg == 0) dst[li][M] = m;
-  };
-  auto common = [&](const uint32_t (&src)[16][4]) {
-    const u32x4v m = *reinterpret_cast<const u32x4v*>(src[li]);
-    return pow2_for(__uint_as_float(max(max(m[0], m[1]), max(m[2], m[3]))));
-  };
-  auto put_state = [&]() {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const Pow2 sc = common(sSm[nt]);
-      sinv[nt] = sc.inv;
-      u32x4v hi, lo;
-      split8(s[nt][0], s[nt][1], sc.s, hi, lo);
-      sS[nt][M][0][lane] = hi;
-      sS[nt][M][1][lane] = lo;
-    }
-  };
-  auto put_own = [&]() {
-    sV[M][lane] = v;
-    if (lane < 16) sFac[M][lane] = fac;
-  };
-  if (nchunks > 0) {
-    load_v(0);
-    load_k(0);
-    load_q(0);
-    load_kp(0, 0);
-    load_kp(0, 1);
-    load_at(0);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) publish(sSm[nt], col_absmax(s[nt]));
-    put_own();
-    load_v(min(1, nchunks - 1));
-    __syncthreads();
-    put_state();
-    __syncthreads();
-  }
-  for (int c = 0; c < nchunks; ++c) {
-    const int cn = min(c + 1, nchunks - 1);
-    // ---- stage A: K_M S, rows 16M+4lg+r, column li of each tile
-    u32x4v sh[NT][4], sl[NT][4];
-    f4v ks[NT], qq[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      ks[nt] = qq[nt] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int bk = 0; bk < 4; ++bk) {
-        sh[nt][bk] = sS[nt][bk][0][lane];
-        sl[nt][bk] = sS[nt][bk][1][lane];
-      }
-    }
-#pragma unroll
-    for (int bk = 0; bk < 4; ++bk)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        ks[nt] = mfma32h(k[bk], sl[nt][bk], ks[nt]);
-        ks[nt] = mfma32h(k[bk], sh[nt][bk], ks[nt]);
-      }
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- stage B: R = beta V - (beta e^g ik) (K S), the next K rows' loads
-    // and Q_M S among it
-    load_k(cn);
-    const f4v c1 = sFac[M][lg], c2 = sFac[M][4 + lg];
-    f4v rv[NT][1];
-    const uint16_t* vs = reinterpret_cast<const uint16_t*>(sV[M]) + 4 * lg * 16 * NT + NT * li;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        rv[nt][0][r] = c1[r] * spk::h2f(vs[16 * NT * r + nt]) - c2[r] * (ks[nt][r] * sinv[nt]);
-#pragma unroll
-    for (int bk = 0; bk < 4; ++bk)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        qq[nt] = mfma32h(q[bk], sl[nt][bk], qq[nt]);
-        qq[nt] = mfma32h(q[bk], sh[nt][bk], qq[nt]);
-      }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 4 * NT, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 2 * NT, 0);
-    }
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) publish(sRm[nt], col_absmax(rv[nt]));
-    __syncthreads();
-    load_q(cn);
-    float rinv[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const Pow2 sc = common(sRm[nt]);
-      rinv[nt] = sc.inv;
-      uint32_t hi[2], lo[2];
-      split2(rv[nt][0][0], rv[nt][0][1], sc.s, hi[0], lo[0]);
-      split2(rv[nt][0][2], rv[nt][0][3], sc.s, hi[1], lo[1]);
-      *reinterpret_cast<uint2*>(reinterpret_cast<char*>(&sR[nt][M >> 1][0][lane]) + 8 * (M & 1)) = make_uint2(hi[0], hi[1]);
-      *reinterpret_cast<uint2*>(reinterpret_cast<char*>(&sR[nt][M >> 1][1][lane]) + 8 * (M & 1)) = make_uint2(lo[0], lo[1]);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 1);
-      __builtin_amdgcn_sched_group_barrier(0x002, 6 * NT, 1);
-    }
-    __syncthreads();
-    // ---- stage D: S <- e^{gL} S + K'^T R
-    u32x4v rh[NT][2], rl[NT][2];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int P = 0; P < 2; ++P) {
-        rh[nt][P] = sR[nt][P][0][lane];
-        rl[nt][P] = sR[nt][P][1][lane];
-      }
-    const f4v sc = sFac[M][12];
-    const f4v qs = sFac[M][8 + lg];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      f4v d[NT];
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) d[nt] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int x = 0; x < 3; ++x)  // lo hi, hi lo, hi hi
-#pragma unroll
-        for (int P = 0; P < 2; ++P)
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            d[nt] = mfma32h(kp[t][P][x == 0 ? 1 : 0], x == 1 ? rl[nt][P] : rh[nt][P], d[nt]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (t == 1) load_kp(cn, 0);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const float f = rinv[nt] * sc[1 + t];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[nt][t][r] = __builtin_fmaf(d[nt][r], f, s[nt][t][r] * sc[0]);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 2);
-      __builtin_amdgcn_sched_group_barrier(0x002, 4 * NT, 2);
-    }
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) publish(sSm[nt], col_absmax(s[nt]));
-    // ---- stage C: o = Qs (Q S) + (A T) R over the pairs P <= M/2; for even M
-    // the pair's second block is above the diagonal and its R is left out
-    // (not multiplied by zero)
-    f4v out[NT], ac[NT];
-    const uint32_t keep = (M & 1) ? 0xffffffffu : 0u;
-    __builtin_amdgcn_sched_barrier(0);
-    load_kp(cn, 1);
-    if (M >= 2) {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        f4v a = {0.f, 0.f, 0.f, 0.f};
-        a = mfma32h(at[0][1], rh[nt][0], a);
-        a = mfma32h(at[0][0], rl[nt][0], a);
-        ac[nt] = mfma32h(at[0][0], rh[nt][0], a);
-        rh[nt][0] = rh[nt][1];
-        rl[nt][0] = rl[nt][1];
-      }
-    } else {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) ac[nt] = f4v{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const u32x4v th = {rh[nt][0][0], rh[nt][0][1], rh[nt][0][2] & keep, rh[nt][0][3] & keep};
-      const u32x4v tl = {rl[nt][0][0], rl[nt][0][1], rl[nt][0][2] & keep, rl[nt][0][3] & keep};
-      f4v a = ac[nt];
-      a = mfma32h(at[1][1], th, a);
-      a = mfma32h(at[1][0], tl, a);
-      a = mfma32h(at[1][0], th, a);
-      const float f = rinv[nt] * sc[3];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        out[nt][r] = __builtin_fmaf(a[r], f, (qq[nt][r] * sinv[nt]) * qs[r]);
-        // formed here, stored below: sunk past the loads, it would keep the
-        // old factors' registers live beside the new ones
-        asm volatile("" : "+v"(out[nt][r]));
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      const int len = min(kC, L - c * kC);
-      const __amdgpu_buffer_rsrc_t orr = __builtin_amdgcn_make_buffer_rsrc(
-          p.core + ((size_t)h * p.core_hs + t_begin + c * kC) * kD, 0, len * kD * 4, kBufDword3);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int off = ((16 * M + 4 * lg + r) * kD + col) * 4;
-        if constexpr (NT == 1) {
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(out[0][r]), orr, off, 0, 0);
-        } else {
-          __builtin_amdgcn_raw_buffer_store_b64(u32x2v{__float_as_uint(out[0][r]), __float_as_uint(out[NT - 1][r])}, orr,
-                                                off, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
-    load_at(cn);
-    put_state();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 3);
-      __builtin_amdgcn_sched_group_barrier(0x002, 8 * NT, 3);
-    }
-    put_own();
-    load_v(min(c + 2, nchunks - 1));
-    __syncthreads();
-  }
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) p.state[st_off + (4 * t + r) * kD + nt] = s[nt][t][r];
 }
 
 __global__ void prefill_collect_kernel(const uint16_t* __restrict__ qkv, const float* __restrict__ gb,
@@ -1694,23 +1203,26 @@ int launch_intra(const ChunkParams& p, int chunks, bool f32, hipStream_t s) {
   return spk::check_launch("spk_chunk_prefill (intra)");
 }
 
-// Value columns per workgroup of the fp16 scan: 32 once 16-column workgroups
-// would number more than two per CU (each operand fetched then serves twice
-// the columns: 8 packed sequences x 16 heads, 1,024 tiles, 0.494 vs 0.673 ms
-// with 16 columns and three workgroups per CU); below that the 16-column
-// tiles keep more CUs busy (one 2048-token sequence: 128 workgroups).
-bool scan_wide(int H, int nseq) { return (long long)kTiles * H * nseq > 2 * 256; }
-
 int launch_scan(const ChunkParams& p, int nseq, bool f32, hipStream_t s) {
   dim3 g((unsigned)(kTiles * p.H * nseq));
-  if (f32 && p.init == nullptr)
-    hipLaunchKernelGGL((chunk_state_kernel<true>), g, dim3(256), 0, s, p);
+  // Three fp16 workgroups per CU (168 VGPRs, a 16-byte spill) only when the
+  // launch has that many workgroups to keep resident; otherwise two per CU
+  // without spilling, with the first-chunk skip when there is no initial
+  // state (that instance's peeled loop spilled more at 168 VGPRs).  Measured,
+  // fp16, 16 heads: one 104-token sequence 9.0 -> 8.0 us; config 2 (1024
+  // workgroups) unchanged either way within noise, so it keeps the old path.
+  const bool z = p.init == nullptr;
+  const bool big = g.x > 2u * 256u;
+  if (f32 && z)
+    hipLaunchKernelGGL((chunk_state_kernel<float, true, 2>), g, dim3(256), 0, s, p);
   else if (f32)
-    hipLaunchKernelGGL((chunk_state_kernel<false>), g, dim3(256), 0, s, p);
-  else if (scan_wide(p.H, nseq))
-    hipLaunchKernelGGL((chunk_scan_split_kernel<2, 2>), dim3(g.x / 2), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((chunk_state_kernel<float, false, 2>), g, dim3(256), 0, s, p);
+  else if (big)
+    hipLaunchKernelGGL((chunk_state_kernel<uint16_t, false, 3>), g, dim3(256), 0, s, p);
+  else if (z)
+    hipLaunchKernelGGL((chunk_state_kernel<uint16_t, true, 2>), g, dim3(256), 0, s, p);
   else
-    hipLaunchKernelGGL((chunk_scan_split_kernel<1, 2>), g, dim3(256), 0, s, p);
+    hipLaunchKernelGGL((chunk_state_kernel<uint16_t, false, 2>), g, dim3(256), 0, s, p);
   return spk::check_launch("spk_chunk_prefill (state)");
 }
 
@@ -1803,13 +1315,6 @@ extern "C" int spk_chunk_prefill(const SpkChunkArgs* a, spk_stream_t stream) {
       co += n;
     }
     std::stable_sort(seqs, seqs + S, [](const SeqEntry& x, const SeqEntry& y) { return x.len > y.len; });
-    // fp16 scan, every workgroup resident from the start (two per CU): the
-    // first 256 workgroups take the longest sequences, one per CU, and the
-    // rest follow shortest first, so that a CU's long scan shares it with a
-    // short one (8 ragged sequences, 512 workgroups: 0.536 -> 0.494 ms)
-    const int per = a->num_heads * kTiles / 2;
-    if (!f32 && scan_wide(a->num_heads, S) && (long long)per * S <= 2 * 256)
-      std::reverse(seqs + std::min(S, (256 + per - 1) / per), seqs + S);
   }
   fill_tables(p, seqs, S);
   if (chunks > 0) {

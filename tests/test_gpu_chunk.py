@@ -423,12 +423,11 @@ def test_padding_rows_never_read_past_the_chunk(dev, oracle, half, last):
         assert max_rel(gs, cs) <= TOL
 
 
-@pytest.mark.parametrize("seqs", [1, 5])  # 16- and 32-column workgroups of the fp16 scan (16 heads)
-def test_fp16_scan_scales_are_per_column(dev, oracle, seqs):
-    """The fp16 scan holds fp32 operands as scaled halves, one power of two per
-    value column: columns of an initial state that differ by 2^80 each keep
-    fp32-level accuracy, and an infinity in V changes nothing in the other
-    columns, in the same column's earlier 16-token blocks, or in other heads."""
+@pytest.mark.parametrize("seqs", [1, 5])  # two and three workgroups of the fp16 scan per CU (16 heads)
+def test_fp16_scan_columns_are_independent(dev, oracle, seqs):
+    """Columns of an initial state that differ by 2^80 each keep fp32-level
+    accuracy, and an infinity in V changes nothing in the other columns, in the
+    same column's earlier 16-token blocks, or in other heads."""
     from spock_amd import synth
     H, T, D = 16, 150, 128
     cu = synth.cu_seqlens_from([T] * seqs)
@@ -440,8 +439,8 @@ def test_fp16_scan_scales_are_per_column(dev, oracle, seqs):
     gc, gs = _run(dev, inp, init=init, cu=cu, half=True)
     sub = {n: np.ascontiguousarray(a[:2, :T]) for n, a in inp.items()}
     c64, s64 = oracle.delta_recurrence_f64(**sub, init=init[0, :2])
-    # the file's 1e-5 against each column's largest value.  Either form's error
-    # here is the decays': a running sum of 64 log-decays below 128 in size
+    # the file's 1e-5 against each column's largest value.  The error here is
+    # the decays': a running sum of 64 log-decays below 128 in size
     # rounds by up to 2^-18 at each step, 8 x 2^-18 x 0.58 = 1.8e-5 (one
     # standard deviation of the sum) at its end in the exponent, where the
     # decayed term itself no longer counts
@@ -459,3 +458,76 @@ def test_fp16_scan_scales_are_per_column(dev, oracle, seqs):
     same = np.ones_like(gs, dtype=bool)
     same[0, 1, :, 37] = False
     assert np.array_equal(bs[same], gs[same])
+
+
+def _fp16_chunk(seed, H=4, T=64):
+    """One chunk of fp16-valued inputs with unit keys and queries.  The
+    log-decays are multiples of 1/16, so that their running sums are exact and
+    the decays add no error of their own."""
+    rng = np.random.default_rng(seed)
+    unit = lambda x: x / np.linalg.norm(x, axis=-1, keepdims=True)
+    inp = {"q": unit(rng.normal(0, 1, (H, T, 128))), "k": unit(rng.normal(0, 1, (H, T, 128))),
+           "v": rng.normal(0, 1, (H, T, 128)),
+           "g": -np.round(np.log1p(np.exp(rng.normal(0, 1, (H, T)))) * 16) / 16,
+           "beta": 1 / (1 + np.exp(-rng.normal(0, 1, (H, T))))}
+    return inp, rng.normal(0, 0.1, (H, 128, 128)).astype(np.float32)
+
+
+def _halves(inp):
+    """The inputs as the call sees them: q, k, v in fp16, g and beta in fp32."""
+    return {n: a.astype(np.float16 if n in "qkv" else np.float32).astype(np.float32) for n, a in inp.items()}
+
+
+@pytest.mark.parametrize("case", ["state-2^26", "state-2^60", "q-1e3", "q-1e4", "v-21", "v-28"])
+def test_fp16_tokens_keep_their_own_precision(dev, oracle, case):
+    """fp32 operands are held element by element: within one chunk, tokens of
+    very different size each come out to fp32 accuracy of their own size -- a
+    large incoming state that decays, query rows of 1e4 beside 1e-4, large early
+    values beside small late ones with a strong decay between them."""
+    inp, init = _fp16_chunk(7)
+    kind, size = case.split("-")
+    if kind == "state":
+        init = init * np.float32(2.0 ** int(size[2:]))
+    elif kind == "q":
+        inp["q"][:, 0::2] *= float(size)
+        inp["q"][:, 1::2] /= float(size)
+    else:
+        inp["v"][:, :32] *= 1e4
+        inp["v"][:, 32:] *= 1e-4
+        inp["g"][:] = 0
+        inp["g"][:, 32] = -float(size)
+        init[:] = 0
+    inp = _halves(inp)
+    gc, gs = _run(dev, inp, init=init[None], half=True)
+    c64, s64 = oracle.delta_recurrence_f64(**inp, init=init)
+    # 2-norm over a token's row and over a state column.  fp32 sums of 128 + 64
+    # products with a 64-step triangular solve before them: the random walk of
+    # 256 roundings is 16 x 2^-24 = 1e-6, and 1e-5 leaves room for the terms
+    # that cancel in one row
+    err = np.linalg.norm(gc - c64, axis=-1) / np.linalg.norm(c64, axis=-1)
+    assert err.max() <= TOL
+    err = np.linalg.norm(gs[0] - s64, axis=1) / np.linalg.norm(s64, axis=1)
+    assert err.max() <= TOL
+
+
+def test_fp16_infinite_query_stays_in_its_row(dev):
+    inp, init = _fp16_chunk(8)
+    inp = _halves(inp)
+    gc, gs = _run(dev, inp, init=init[None], half=True)
+    inp["q"][1, 0, 3] = inp["q"][1, 16, 5] = inp["q"][1, 41, 7] = np.inf
+    bc, bs = _run(dev, inp, init=init[None], half=True)
+    hit = [0, 16, 41]
+    assert not np.isfinite(bc[1, hit]).any()
+    same = np.ones(gc.shape[:2], dtype=bool)
+    same[1, hit] = False
+    assert np.array_equal(bc[same], gc[same]) and np.array_equal(bs, gs)
+
+
+def test_fp16_infinite_value_stays_infinite(dev):
+    """An infinite value reaches the chunk's later tokens and the state as
+    infinities (no NaN: there is nothing that cancels it)."""
+    inp, init = _fp16_chunk(9)
+    inp = _halves(inp)
+    inp["v"][1, 20, 7] = np.inf
+    bc, bs = _run(dev, inp, init=init[None], half=True)
+    assert np.isinf(bc[1, 20:, 7]).all() and np.isinf(bs[0, 1, :, 7]).all()
