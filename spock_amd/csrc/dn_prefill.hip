@@ -59,7 +59,10 @@ __global__ __launch_bounds__(256) void dn_prefill_conv_kernel(const uint16_t* __
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int j = T - 4 + i;
-        last[half][i] = j >= 0 ? qkv[(long long)j * ld + ch] : ov[min(j + 4, 3)];
+        // before row 0: ov[T + i], selected (an index that depends on T would
+        // put ov on the stack)
+        const uint16_t before = T == 1 ? ov[min(i + 1, 3)] : T == 2 ? ov[min(i + 2, 3)] : ov[3];
+        last[half][i] = j >= 0 ? qkv[(long long)j * ld + ch] : before;
       }
 #pragma unroll
       for (int i = 0; i < 3; ++i) raw[half][i] = ov[i + 1];  // rows -3 .. -1
