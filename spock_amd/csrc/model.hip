@@ -1265,6 +1265,7 @@ __global__ __launch_bounds__(256) void rmsnorm256_kernel(const uint16_t* __restr
 
 // VEC: 8 elements per thread and turn (16-byte aligned rows); the rest of n one
 // by one.
+constexpr long long kSiluVecMin = 512 * 3584;
 template <bool VEC>
 __global__ void silu_gate_kernel(const uint16_t* g, const uint16_t* u, uint16_t* y, long long n) {
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
@@ -2068,9 +2069,12 @@ extern "C" int spk_silu_gate_f16(const uint16_t* g, const uint16_t* u, uint16_t*
   if (!g || !u || !y) return spk::fail(SPK_ERR_NULL, "spk_silu_gate_f16: NULL pointer");
   if (n <= 0) return spk::fail(SPK_ERR_SHAPE, "spk_silu_gate_f16: n %lld", (long long)n);
   hipStream_t s = spk::to_hip(stream);
-  // 8 elements per thread where the rows are aligned (2,000 x 3,584 values: 13.6
-  // -> 9.8 us; one by one, an access of 16 bytes took 8 load instructions)
-  if (n >= 8 && spk::aligned(g, 16) && spk::aligned(u, 16) && spk::aligned(y, 16))
+  // 8 elements per thread where the rows are aligned and one by one would take
+  // several turns of the grid.  In microseconds for rows of 3,584, one by one ->
+  // eight at a time: 1 row 1.80 -> 2.14, 128 2.18 -> 2.47, 256 2.80 -> 2.79, 448
+  // 3.53 -> 3.65, 512 3.77 -> 3.73, 1,024 5.9 -> 5.3, 2,000 13.2 -> 9.5 (a lane's
+  // eight values are formed one after the other, which a short call waits for)
+  if (n >= kSiluVecMin && spk::aligned(g, 16) && spk::aligned(u, 16) && spk::aligned(y, 16))
     hipLaunchKernelGGL((silu_gate_kernel<true>), dim3(grid_for((n + 7) / 8)), dim3(256), 0, s, g, u, y, (long long)n);
   else
     hipLaunchKernelGGL((silu_gate_kernel<false>), dim3(grid_for(n)), dim3(256), 0, s, g, u, y, (long long)n);

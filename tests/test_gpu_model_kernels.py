@@ -415,7 +415,8 @@ def test_elementwise_gates_bitexact(dev):
     assert np.array_equal(_u16(y2), e2)
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9, 4097])
+# one by one, and from 1,835,008 values on eight at a time with a rest
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 4097, 1835007, 1835008, 1835017])
 @pytest.mark.parametrize("shift", [0, 1])  # 16-byte aligned rows, and not
 def test_silu_gate_in_place_any_length_and_alignment(dev, n, shift):
     from spock_amd import _lib
