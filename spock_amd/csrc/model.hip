@@ -1218,12 +1218,15 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
 // RMSNorm(1+w) of rows of 1024, one wave per row: lane l holds the partials of
 // threads l, l + 64, l + 128 and l + 192 of rms_norm.comp (4 contiguous squares
 // each), so its tree's first two levels are the lane's own and the rest stay in
-// registers -- no LDS, no barrier, a quarter of the workgroups (512 rows: 3.9 ->
-// 3.1 us in a DeltaNet layer's prefill, 2,000 rows 5.3 -> 5.1).
+// registers -- no LDS, no barrier (512 rows: 3.9 -> 3.1 us in a DeltaNet
+// layer's prefill, 2,000 rows 5.3 -> 5.1).  Four rows per workgroup; where that
+// leaves most CUs without one, a row each (back to back, in microseconds, four ->
+// one per workgroup: 16 rows 1.91 -> 1.77, 128 1.94 -> 1.79, 256 1.92 -> 1.92).
+constexpr int kRmsSpread = 256;
 __global__ __launch_bounds__(256) void rmsnorm1024_kernel(const uint16_t* __restrict__ x,
                                                           const uint16_t* __restrict__ w,
                                                           uint16_t* __restrict__ y, int rows) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= rows) return;
   const size_t base = (size_t)row * kHidden + 4 * lane;
   float v[4][4], wf[4][4], p[4];
@@ -2058,7 +2061,9 @@ extern "C" int spk_rmsnorm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y
   if (!spk::aligned(x, 8) || !spk::aligned(w, 8) || !spk::aligned(y, 8))
     return spk::fail(SPK_ERR_ALIGN, "spk_rmsnorm_f16: 8-byte alignment required");
   hipStream_t s = spk::to_hip(stream);
-  if (n == kHidden)
+  if (n == kHidden && rows < kRmsSpread)
+    hipLaunchKernelGGL(rmsnorm1024_kernel, dim3(rows), dim3(64), 0, s, x, w, y, rows);
+  else if (n == kHidden)
     hipLaunchKernelGGL(rmsnorm1024_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, x, w, y, rows);
   else
     hipLaunchKernelGGL(rmsnorm256_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, x, w, y, rows);

@@ -380,7 +380,8 @@ def test_attention_decode_position_out_of_range_writes_nothing(dev):
     assert not _u16(d["out"]).any()
 
 
-@pytest.mark.parametrize("n,rows", [(1024, 7), (256, 13)])
+# rows of 1024: one per workgroup, four from 256 rows on (the last one in part)
+@pytest.mark.parametrize("n,rows", [(1024, 7), (256, 13), (1024, 1), (1024, 255), (1024, 256), (1024, 259)])
 def test_rmsnorm_rows_bitexact(dev, n, rows):
     from spock_amd import _lib
     x = _rand16(30 + n, rows * n)
