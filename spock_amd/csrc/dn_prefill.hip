@@ -143,12 +143,16 @@ __device__ __forceinline__ void norm_gate_row(float oa, float ob, const uint16_t
   }
 }
 
-// Gated RMSNorm of the fp32 chunk output: grid (4, T); wave = head.
+// Gated RMSNorm of the fp32 chunk output: wave = head, four waves per workgroup
+// from kGateSpread tokens on, below one (back to back, in microseconds, one ->
+// four: 4 tokens 2.03 -> 2.06, 16 2.05 -> 2.08, 96 2.35 -> 2.19, 512 4.6 -> 3.9,
+// 2,000 11.3 -> 9.6).
+constexpr int kGateSpread = 48;
 __global__ __launch_bounds__(256) void dn_norm_gate_kernel(const float* __restrict__ core, long long head_stride,
                                                           const uint16_t* __restrict__ z, long long zld,
                                                           const float* __restrict__ norm_w, float eps,
                                                           uint16_t* __restrict__ out, long long old) {
-  const int h = blockIdx.x * 4 + (threadIdx.x >> 6), t = blockIdx.y, lane = threadIdx.x & 63;
+  const int h = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), t = blockIdx.y, lane = threadIdx.x & 63;
   const float* o = core + ((long long)h * head_stride + t) * kDim;
   norm_gate_row(o[lane], o[lane + 64], z + (long long)t * zld + h * kDim, norm_w, eps,
                 out + (long long)t * old + h * kDim, lane);
@@ -203,7 +207,8 @@ extern "C" int spk_deltanet_norm_gate(const float* core, int64_t core_head_strid
   if (tokens <= 0 || core_head_stride < tokens || z_ld < kHeads * kDim || out_ld < kHeads * kDim)
     return spk::fail(SPK_ERR_SHAPE, "spk_deltanet_norm_gate: tokens %d head stride %lld", tokens,
                      (long long)core_head_stride);
-  hipLaunchKernelGGL(dn_norm_gate_kernel, dim3(kHeads / 4, tokens), dim3(256), 0, spk::to_hip(stream), core,
+  const int waves = tokens < kGateSpread ? 1 : 4;
+  hipLaunchKernelGGL(dn_norm_gate_kernel, dim3(kHeads / waves, tokens), dim3(64 * waves), 0, spk::to_hip(stream), core,
                      (long long)core_head_stride, z, (long long)z_ld, norm_weight, eps != 0.0f ? eps : 1e-6f, out,
                      (long long)out_ld);
   return spk::check_launch("spk_deltanet_norm_gate");

@@ -474,9 +474,10 @@ def test_deltanet_prefill_conv_bitexact(dev, oracle, T):
         assert np.array_equal(got, want), ["q", "k", "v"][j]
 
 
-def test_deltanet_prefill_gbeta_and_norm_gate_bitexact(dev, oracle):
+@pytest.mark.parametrize("T", [37, 47, 48])  # one wave per workgroup of the norm gate, four from 48 tokens on
+def test_deltanet_prefill_gbeta_and_norm_gate_bitexact(dev, oracle, T):
     from spock_amd import _lib
-    T, layer = 37, 2
+    layer = 2
     a, b = _rand16(70, T * 16), _rand16(71, T * 16)
     alb = np.stack([np.linspace(-1, 1, 3 * 16, dtype=np.float32),
                     oracle.h2f(_rand16(72, 3 * 16, 0.1))], -1).astype(np.float32)
