@@ -342,13 +342,15 @@ def test_attention_prefill_bitexact(dev, pos0, T):
 
 # the matrix-core tiles (192 tokens and 150 score workgroups up): whole and part
 # tiles, starts on and off tile and block edges, a block seen by part of a tile
-@pytest.mark.parametrize("pos0,T", [(0, 385), (0, 400), (61, 335), (190, 256), (48, 337), (300, 192), (305, 199)])
+# and past 16 blocks (1,024 positions), where a row's maximum takes more than one turn
+@pytest.mark.parametrize("pos0,T", [(0, 385), (0, 400), (61, 335), (190, 256), (48, 337), (300, 192), (305, 199),
+                                    (900, 200), (1017, 195), (2040, 193)])
 def test_attention_prefill_tiles_bitexact(dev, pos0, T):
     """The matrix-core path against the oracle, bit for bit; then the same with
     one value of V infinite: rows that may not see it are unchanged."""
     from spock_amd import _lib
     print(f"[attention prefill tiles pos0={pos0} T={T}]", flush=True)
-    max_seq = 640
+    max_seq = max(640, pos0 + T + 7)
     rope, kv, qg, k, v, qn, kn = _attn_inputs(300 + T, max_seq, pos0, T)
     kv[(pos0 + T) * 1024:] = 0x7E00  # rows past the prompt (NaN) are not read
     for inf_at in (None, T - 9):
@@ -364,6 +366,42 @@ def test_attention_prefill_tiles_bitexact(dev, pos0, T):
         assert np.array_equal(np.isnan(got), np.isnan(exp))
         ok = ~np.isnan(exp)
         assert np.array_equal(got[ok].view(np.uint16), exp[ok].view(np.uint16))
+
+
+@pytest.mark.parametrize("what", ["k-cache-inf", "k-cache-nan", "k-late", "q", "v-late"])
+def test_attention_prefill_tiles_non_finite_rows(dev, what):
+    """Infinities and NaN on the matrix-core path against the block kernel, which
+    the same tokens take in calls of at most 128: the same bits, NaN in the same
+    places.  In the cache every row sees them; a late token's only some rows of a
+    tile may see."""
+    from spock_amd import _lib
+    print(f"[attention prefill tiles {what}]", flush=True)
+    pos0, T, max_seq = 100, 327, 640
+    rope, kv, qg, k, v, qn, kn = _attn_inputs(900, max_seq, pos0, T)
+    if what.startswith("k-cache"):
+        kv[50 * 1024 + 3] = 0x7C00 if what == "k-cache-inf" else 0x7E00
+    elif what == "k-late":
+        k[(T - 9) * 512 + 3] = 0x7C00
+    elif what == "q":
+        qg[200 * 4096 + 512 + 9] = 0x7C00
+    else:
+        v[(T - 9) * 512 + 300] = 0x7E00
+    a, d = _attn_args(dev, rope, kv, qg, k, v, qn, kn, max_seq, T, pos0 + T)
+    _lib.check(_lib.lib().spk_attention_prefill(C.byref(a), pos0, T, _stream()), "spk_attention_prefill")
+    outs, kv2 = [], _h(kv, dev)
+    for t in range(0, T, 128):
+        n = min(128, T - t)
+        b, e = _attn_args(dev, rope, kv, qg[t * 4096:(t + n) * 4096], k[t * 512:(t + n) * 512], v[t * 512:(t + n) * 512],
+                          qn, kn, max_seq, n, pos0 + t + n)
+        b.kv_cache = kv2.data_ptr()
+        _lib.check(_lib.lib().spk_attention_prefill(C.byref(b), pos0 + t, n, _stream()), "spk_attention_prefill")
+        torch.cuda.synchronize()
+        outs.append(_u16(e["out"]))
+    exp, got = np.concatenate(outs).view(np.float16), _u16(d["out"]).view(np.float16)
+    assert np.array_equal(_u16(d["kv"]), _u16(kv2))
+    bad = np.isnan(exp)
+    assert np.array_equal(np.isnan(got), bad) and bad.any() and not bad.all()
+    assert np.array_equal(got[~bad].view(np.uint16), exp[~bad].view(np.uint16))
 
 
 def test_attention_decode_position_out_of_range_writes_nothing(dev):
