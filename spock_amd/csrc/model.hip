@@ -794,9 +794,10 @@ __global__ __launch_bounds__(256) void attn_prefill_blocks_kernel(AttnArgs a) {
 //                          blocks' partial outputs stay in registers instead of
 //                          going through memory (1 KB per token, head and
 //                          block; the weights are 256 B)
-// Bound by the matrix issue of 32 cycles per instruction (2,000 tokens: 56 us of
-// it in each of the last two launches, which take 106 and 127 us), by the
-// score launches' prologues and by the longest tile's chain of blocks.
+// Bound by the matrix issue of 32 cycles per instruction (2,000 tokens: 54 us of
+// it at 2.4 GHz in each of the last two launches, which take 101 and 122 us;
+// 1,000 tokens: 38 and 44 us, matrix cores 32% and 27% busy), by the score
+// launches' prologues and by the longest tile's chain of blocks.
 // Attention layer prefill, projections included: 512 tokens 122 -> 89 us, 1,000
 // 318 -> 136, 2,000 1,108 -> 318, 500 at position 1,000 251 -> 141.
 // ---------------------------------------------------------------------------
